@@ -111,8 +111,9 @@ struct DevState {
     // (the fused schedule's node passes; see xcd_block)
     int rev;
     // elements whose Mohr-Coulomb return is left to the return kernel of the
-    // fused schedule: count, element ids, and per entry the trial stress and
-    // the stress trace before the update (8 doubles)
+    // fused schedule, in segments of 64 (element e's is e / 64): each
+    // segment's count, element ids, and per entry the trial stress and the
+    // stress trace before the update (8 doubles)
     int *ret_count, *ret_elem;
     double *ret_val;
     MixedRet *ret_mix;                            // the mixed-precision schedule's records
@@ -637,13 +638,15 @@ __device__ __forceinline__ void dsyevc3(const double A[3][3], double w[3])
 }
 
 // Householder tridiagonalisation (3x3-C/dsytrd3.c:28-104)
-__device__ __noinline__ void dsytrd3(const double A[3][3], double Q[3][3], double d[3], double e[2])
+__device__ __forceinline__ void dsytrd3(const double A[3][3], double Q[3][3], double d[3], double e[2])
 {
     const int n = 3;
     double u[3], q[3];
     double omega, f, K, h, g;
+#pragma unroll
     for (int i = 0; i < n; i++) {
         Q[i][i] = 1.0;
+#pragma unroll
         for (int j = 0; j < i; j++) Q[i][j] = Q[j][i] = 0.0;
     }
     h = DES_SQR(A[0][1]) + DES_SQR(A[0][2]);
@@ -657,79 +660,105 @@ __device__ __noinline__ void dsytrd3(const double A[3][3], double Q[3][3], doubl
     if (omega > 0.0) {
         omega = 1.0 / omega;
         K = 0.0;
+#pragma unroll
         for (int i = 1; i < n; i++) {
             f = A[1][i] * u[1] + A[i][2] * u[2];
             q[i] = omega * f;
             K += u[i] * f;
         }
         K *= 0.5 * DES_SQR(omega);
+#pragma unroll
         for (int i = 1; i < n; i++) q[i] = q[i] - K * u[i];
         d[0] = A[0][0];
         d[1] = A[1][1] - 2.0 * q[1] * u[1];
         d[2] = A[2][2] - 2.0 * q[2] * u[2];
+#pragma unroll
         for (int j = 1; j < n; j++) {
             f = omega * u[j];
+#pragma unroll
             for (int i = 1; i < n; i++) Q[i][j] = Q[i][j] - f * u[i];
         }
         e[1] = A[1][2] - q[1] * u[2] - u[1] * q[2];
     } else {
+#pragma unroll
         for (int i = 0; i < n; i++) d[i] = A[i][i];
         e[1] = A[1][2];
     }
 }
 
-// QL with implicit shifts, at most 30 sweeps per eigenvalue (3x3-C/dsyevq3.c:29-134)
-__device__ __noinline__ int dsyevq3(const double A[3][3], double Q[3][3], double w[3])
+// one plane rotation of a QL sweep (the loop body of 3x3-C/dsyevq3.c:78-120),
+// between rows i and i + 1; e2 is what the loop stores in e[i + 1]
+template <int I> __device__ __forceinline__ void dsyevq3_rotate(double Q[3][3], double w[3], double ei, double &e2,
+                                                                double &g, double &s, double &c, double &p)
 {
-    const int n = 3;
-    double e[3];
-    double g, r, p, f, b, s, c, t;
-    int nIter, m;
+    double f = s * ei, r;
+    const double b = c * ei;
+    if (fabs(f) > fabs(g)) {
+        c = g / f;
+        r = sqrt(DES_SQR(c) + 1.0);
+        e2 = f * r;
+        c *= (s = 1.0 / r);
+    } else {
+        s = f / g;
+        r = sqrt(DES_SQR(s) + 1.0);
+        e2 = g * r;
+        s *= (c = 1.0 / r);
+    }
+    g = w[I + 1] - p;
+    r = (w[I] - g) * s + 2.0 * c * b;
+    p = s * r;
+    w[I + 1] = g + p;
+    g = c * r - b;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const double t = Q[k][I + 1];
+        Q[k][I + 1] = s * Q[k][I] + c * t;
+        Q[k][I] = c * Q[k][I] - s * t;
+    }
+}
+
+// QL with implicit shifts, at most 30 sweeps per eigenvalue
+// (3x3-C/dsyevq3.c:29-134), the loops over the three rows written out so that
+// every index is a constant: the matrices stay in registers (with variable
+// indices they were 224 bytes of scratch a lane for every return, also for
+// the ones that never come here)
+__device__ __forceinline__ int dsyevq3(const double A[3][3], double Q[3][3], double w[3])
+{
+    double e[2], unused;
+    double g, r, p, s, c;
     dsytrd3(A, Q, w, e);
-    for (int l = 0; l < n - 1; l++) {
-        nIter = 0;
-        while (1) {
-            for (m = l; m <= n - 2; m++) {
-                g = fabs(w[m]) + fabs(w[m + 1]);
-                if (fabs(e[m]) + g == g) break;
-            }
-            if (m == l) break;
-            if (nIter++ >= 30) return -1;
-            g = (w[l + 1] - w[l]) / (e[l] + e[l]);
-            r = sqrt(DES_SQR(g) + 1.0);
-            if (g > 0) g = w[m] - w[l] + e[l] / (g + r);
-            else g = w[m] - w[l] + e[l] / (g - r);
-            s = c = 1.0;
-            p = 0.0;
-            for (int i = m - 1; i >= l; i--) {
-                f = s * e[i];
-                b = c * e[i];
-                if (fabs(f) > fabs(g)) {
-                    c = g / f;
-                    r = sqrt(DES_SQR(c) + 1.0);
-                    e[i + 1] = f * r;
-                    c *= (s = 1.0 / r);
-                } else {
-                    s = f / g;
-                    r = sqrt(DES_SQR(s) + 1.0);
-                    e[i + 1] = g * r;
-                    s *= (c = 1.0 / r);
-                }
-                g = w[i + 1] - p;
-                r = (w[i] - g) * s + 2.0 * c * b;
-                p = s * r;
-                w[i + 1] = g + p;
-                g = c * r - b;
-                for (int k = 0; k < n; k++) {
-                    t = Q[k][i + 1];
-                    Q[k][i + 1] = s * Q[k][i] + c * t;
-                    Q[k][i] = c * Q[k][i] - s * t;
-                }
-            }
-            w[l] -= p;
-            e[l] = g;
-            e[m] = 0.0;
-        }
+    for (int it = 0;; it++) {                   // l = 0
+        g = fabs(w[0]) + fabs(w[1]);
+        if (fabs(e[0]) + g == g) break;
+        g = fabs(w[1]) + fabs(w[2]);
+        const bool two = !(fabs(e[1]) + g == g);        // m == 2, else m == 1
+        if (it >= 30) return -1;
+        g = (w[1] - w[0]) / (e[0] + e[0]);
+        r = sqrt(DES_SQR(g) + 1.0);
+        const double wm = two ? w[2] : w[1];
+        if (g > 0) g = wm - w[0] + e[0] / (g + r);
+        else g = wm - w[0] + e[0] / (g - r);
+        s = c = 1.0;
+        p = 0.0;
+        if (two) dsyevq3_rotate<1>(Q, w, e[1], unused, g, s, c, p);
+        dsyevq3_rotate<0>(Q, w, e[0], e[1], g, s, c, p);
+        w[0] -= p;
+        e[0] = g;
+        if (!two) e[1] = 0.0;                   // e[m] = 0
+    }
+    for (int it = 0;; it++) {                   // l = 1
+        g = fabs(w[1]) + fabs(w[2]);
+        if (fabs(e[1]) + g == g) break;
+        if (it >= 30) return -1;
+        g = (w[2] - w[1]) / (e[1] + e[1]);
+        r = sqrt(DES_SQR(g) + 1.0);
+        if (g > 0) g = w[2] - w[1] + e[1] / (g + r);
+        else g = w[2] - w[1] + e[1] / (g - r);
+        s = c = 1.0;
+        p = 0.0;
+        dsyevq3_rotate<1>(Q, w, e[1], unused, g, s, c, p);
+        w[1] -= p;
+        e[1] = g;
     }
     return 0;
 }
@@ -752,20 +781,26 @@ __device__ __forceinline__ int dsyevh3(const double A[3][3], double Q[3][3], dou
     Q[1][0] = Q[1][1] + A[1][2] * w[0];
     Q[2][0] = (A[0][0] - w[0]) * (A[1][1] - w[0]) - Q[2][1];
     norm = DES_SQR(Q[0][0]) + DES_SQR(Q[1][0]) + DES_SQR(Q[2][0]);
-    if (norm <= error) return dsyevq3(A, Q, w);
-    norm = sqrt(1.0 / norm);
-    for (int j = 0; j < 3; j++) Q[j][0] = Q[j][0] * norm;
-    Q[0][1] = Q[0][1] + A[0][2] * w[1];
-    Q[1][1] = Q[1][1] + A[1][2] * w[1];
-    Q[2][1] = (A[0][0] - w[1]) * (A[1][1] - w[1]) - Q[2][1];
-    norm = DES_SQR(Q[0][1]) + DES_SQR(Q[1][1]) + DES_SQR(Q[2][1]);
-    if (norm <= error) return dsyevq3(A, Q, w);
-    norm = sqrt(1.0 / norm);
-    for (int j = 0; j < 3; j++) Q[j][1] = Q[j][1] * norm;
-    Q[0][2] = Q[1][0] * Q[2][1] - Q[2][0] * Q[1][1];
-    Q[1][2] = Q[2][0] * Q[0][1] - Q[0][0] * Q[2][1];
-    Q[2][2] = Q[0][0] * Q[1][1] - Q[1][0] * Q[0][1];
-    return 0;
+    bool ql = norm <= error;
+    if (!ql) {
+        norm = sqrt(1.0 / norm);
+#pragma unroll
+        for (int j = 0; j < 3; j++) Q[j][0] = Q[j][0] * norm;
+        Q[0][1] = Q[0][1] + A[0][2] * w[1];
+        Q[1][1] = Q[1][1] + A[1][2] * w[1];
+        Q[2][1] = (A[0][0] - w[1]) * (A[1][1] - w[1]) - Q[2][1];
+        norm = DES_SQR(Q[0][1]) + DES_SQR(Q[1][1]) + DES_SQR(Q[2][1]);
+        ql = norm <= error;
+        if (!ql) {
+            norm = sqrt(1.0 / norm);
+#pragma unroll
+            for (int j = 0; j < 3; j++) Q[j][1] = Q[j][1] * norm;
+            Q[0][2] = Q[1][0] * Q[2][1] - Q[2][0] * Q[1][1];
+            Q[1][2] = Q[2][0] * Q[0][1] - Q[0][0] * Q[2][1];
+            Q[2][2] = Q[0][0] * Q[1][1] - Q[1][0] * Q[0][1];
+        }
+    }
+    return ql ? dsyevq3(A, Q, w) : 0;
 }
 
 // principal_stresses3 (rheology.cxx:13-68): eigenpairs in ascending order
