@@ -48,14 +48,15 @@ inline int nblocks(long n) { return (int)((n + BLOCK - 1) / BLOCK); }
 // the top down: a pass that follows one walking upwards starts where that one
 // ended, on the lines it wrote last, which are still in the L2 and the 256 MB
 // Infinity Cache when the pass's data are larger than both.
-__device__ __forceinline__ int xcd_block(int rev = 0)
+__device__ __forceinline__ int xcd_block_of(int nb, int rev)
 {
-    const int nb = gridDim.x, b = blockIdx.x;
+    const int b = blockIdx.x;
     const int q = nb >> 3, r = nb & 7, x = b & 7;
     int j = b >> 3;
     if (rev) j = q + (x < r ? 1 : 0) - 1 - j;    // XCD x has q (+1 if x < r) blocks
     return x * q + min(x, r) + j;
 }
+__device__ __forceinline__ int xcd_block(int rev = 0) { return xcd_block_of(gridDim.x, rev); }
 
 // Element / node index of this thread.  For batched models the block's model
 // supplies the parameters and scalars (the kernel's by-value DevState is
@@ -179,6 +180,34 @@ template <int ND> __device__ __forceinline__ void bind_model(DevState &s, int m)
     s.edge_valid = s.evvb + m * (DES_NBDRY * DES_NBDRY);
 }
 
+// Sums over node n's list in its (ascending host element) order: load(entry, v)
+// gives the K terms of an entry.  DEPTH entries are requested together and the
+// last, ragged round like the others (its missing entries repeat the last one
+// and are not added), so a list of 24 costs three round trips to memory.  One
+// entry at a time, in blocks of 256 threads, the node sums of a 100 k-tet model
+// took 12-16 us each; eight at a time in blocks of 64 (one wavefront per CU at
+// that size) 5.5-7 us, and k_mass_node of 8.09 M tets 1034 -> 234 us.
+constexpr int NODE_BLOCK = 64;
+template <int K, int DEPTH = 8, class Load>
+__device__ __forceinline__ void list_sums(const DevState &s, int n, double (&sum)[K], Load &&load)
+{
+#pragma unroll
+    for (int k = 0; k < K; ++k) sum[k] = 0;
+    const int p1 = s.csr_off[n + 1];
+    for (int p = s.csr_off[n]; p < p1; p += DEPTH) {
+        int en[DEPTH];
+        double v[DEPTH][K];
+#pragma unroll
+        for (int j = 0; j < DEPTH; ++j) en[j] = s.csr_ent[min(p + j, p1 - 1)];
+#pragma unroll
+        for (int j = 0; j < DEPTH; ++j) load(en[j], v[j]);
+#pragma unroll
+        for (int j = 0; j < DEPTH; ++j)
+#pragma unroll
+            for (int k = 0; k < K; ++k) sum[k] = p + j < p1 ? sum[k] + v[j][k] : sum[k];
+    }
+}
+
 // compute_volume (geometry.cxx:86-108)
 template <int ND> __global__ __launch_bounds__(BLOCK) void k_volume(DevState s)
 {
@@ -231,6 +260,13 @@ template <int ND> __device__ __forceinline__ void mass_of(const DevState &s, int
     tm = rho_e * arithmetic_mean(s, P->heat_capacity, e) * vol / NPE;
 }
 
+// m and tm of every element side by side (escal's second half): the node sums
+// gather both with one 16-byte load
+__device__ __forceinline__ double2 *mass_terms(const DevState &s)
+{
+    return reinterpret_cast<double2 *>(s.escal + 2 * (long)s.E);
+}
+
 template <int ND> __global__ __launch_bounds__(BLOCK) void k_mass_elem(DevState s)
 {
     BIND_ELEM(s, e);
@@ -238,26 +274,24 @@ template <int ND> __global__ __launch_bounds__(BLOCK) void k_mass_elem(DevState 
     load_conn<ND>(s, e, c);
     double m, tm;
     mass_of<ND>(s, e, s.volume[e], elem_mean<ND>(s.T, c), m, tm);
-    s.escal[1 * (long)s.E + e] = m;
-    s.escal[2 * (long)s.E + e] = tm;
+    mass_terms(s)[e] = make_double2(m, tm);
 }
 
 // node part of compute_mass (geometry.cxx:353-359)
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_mass_node(DevState s)
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_mass_node(DevState s)
 {
-    BIND_NODE(s, n);
-    constexpr int NPE = Dim<ND>::NPE;
-    const int thermal = s.P->has_thermal_diffusion;
-    double vn = 0, m = 0, tm = 0;
-    for (int p = s.csr_off[n]; p < s.csr_off[n + 1]; ++p) {
-        int e = s.csr_ent[p] / NPE;
-        vn += s.volume[e];
-        m += s.escal[1 * (long)s.E + e];
-        if (thermal) tm += s.escal[2 * (long)s.E + e];
-    }
-    s.volume_n[n] = vn;
-    s.mass[n] = m;
-    s.tmass[n] = tm;
+    BIND_NODE_NB(s, n, NODE_BLOCK);
+    double sum[3];
+    list_sums(s, n, sum, [&](int ent, double *v) {
+        const int e = ent / Dim<ND>::NPE;
+        const double2 mt = mass_terms(s)[e];
+        v[0] = s.volume[e];
+        v[1] = mt.x;
+        v[2] = mt.y;
+    });
+    s.volume_n[n] = sum[0];
+    s.mass[n] = sum[1];
+    s.tmass[n] = s.P->has_thermal_diffusion ? sum[2] : 0.0;
 }
 
 // thermal contribution of element e to tdot at its nodes (fields.cxx:110-142)
@@ -287,19 +321,26 @@ template <int ND> __device__ __forceinline__ void temperature_contrib(const DevS
     }
 }
 
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_temp_elem(DevState s)
+template <int ND> __device__ __forceinline__ void temp_elem(const DevState &s, int e, const int *c,
+                                                          const double sh[ND][Dim<ND>::NPE])
 {
-    BIND_ELEM(s, e);
     constexpr int NPE = Dim<ND>::NPE;
-    int c[NPE];
-    load_conn<ND>(s, e, c);
-    double sh[ND][NPE], Tn[NPE], out[NPE];
-    load_shp<ND>(s, e, sh);
+    double Tn[NPE], out[NPE];
 #pragma unroll
     for (int i = 0; i < NPE; ++i) Tn[i] = s.T[c[i]];
     temperature_contrib<ND>(s, e, s.volume[e], sh, Tn, out);
 #pragma unroll
     for (int i = 0; i < NPE; ++i) s.ework[e * NPE + i] = out[i];
+}
+
+template <int ND> __global__ __launch_bounds__(BLOCK) void k_temp_elem(DevState s)
+{
+    BIND_ELEM(s, e);
+    int c[Dim<ND>::NPE];
+    load_conn<ND>(s, e, c);
+    double sh[ND][Dim<ND>::NPE];
+    load_shp<ND>(s, e, sh);
+    temp_elem<ND>(s, e, c, sh);
 }
 
 // temperature update with its boundary conditions (fields.cxx:153-162)
@@ -318,56 +359,68 @@ __device__ __forceinline__ double temperature_new(const DevState &s, int n, doub
     return temperature_new_f(s, s.bcflag[n], T, tdot, dt, tmass);
 }
 
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_temp_node(DevState s)
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_temp_node(DevState s)
 {
-    BIND_NODE(s, n);
-    double tdot = 0;
-    for (int p = s.csr_off[n]; p < s.csr_off[n + 1]; ++p) tdot += s.ework[s.csr_ent[p]];
-    s.ntmp[n] = tdot;
-    s.T[n] = temperature_new(s, n, s.T[n], tdot, s.sc->dt, s.tmass[n]);
+    BIND_NODE_NB(s, n, NODE_BLOCK);
+    double tdot[1];
+    list_sums(s, n, tdot, [&](int ent, double *v) { v[0] = s.ework[ent]; });
+    s.ntmp[n] = tdot[0];
+    s.T[n] = temperature_new(s, n, s.T[n], tdot[0], s.sc->dt, s.tmass[n]);
+}
+
+// update_strain_rate; returns tr(edot)
+template <int ND> __device__ __forceinline__ double strain_rate_elem(const DevState &s, int e, const int *c,
+                                                                   const double sh[ND][Dim<ND>::NPE])
+{
+    constexpr int NPE = Dim<ND>::NPE, NSTR = Dim<ND>::NSTR;
+    double v[NPE][ND], sr[NSTR];
+    gather_vec<ND>(s.vel, s.N, c, v);
+    strain_rate<ND>(v, sh, sr);
+#pragma unroll
+    for (int k = 0; k < NSTR; ++k) s.strain_rate[k * (long)s.E + e] = sr[k];
+    return trace<ND>(sr);
 }
 
 template <int ND> __global__ __launch_bounds__(BLOCK) void k_strain_rate(DevState s)
 {
     BIND_ELEM(s, e);
-    constexpr int NPE = Dim<ND>::NPE, NSTR = Dim<ND>::NSTR;
-    int c[NPE];
+    int c[Dim<ND>::NPE];
     load_conn<ND>(s, e, c);
-    double v[NPE][ND], sh[ND][NPE], sr[NSTR];
-    gather_vec<ND>(s.vel, s.N, c, v);
+    double sh[ND][Dim<ND>::NPE];
     load_shp<ND>(s, e, sh);
-    strain_rate<ND>(v, sh, sr);
-#pragma unroll
-    for (int k = 0; k < NSTR; ++k) s.strain_rate[k * (long)s.E + e] = sr[k];
+    strain_rate_elem<ND>(s, e, c, sh);
 }
 
 // compute_dvoldt (geometry.cxx:111-155), into ntmp
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_dvoldt_node(DevState s)
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_dvoldt_node(DevState s)
 {
-    BIND_NODE(s, n);
-    constexpr int NPE = Dim<ND>::NPE;
-    double sum = 0;
-    for (int p = s.csr_off[n]; p < s.csr_off[n + 1]; ++p) {
-        int e = s.csr_ent[p] / NPE;
+    BIND_NODE_NB(s, n, NODE_BLOCK);
+    double sum[1];
+    list_sums(s, n, sum, [&](int ent, double *v) {
+        const int e = ent / Dim<ND>::NPE;
         double sr[ND];
 #pragma unroll
         for (int k = 0; k < ND; ++k) sr[k] = s.strain_rate[k * (long)s.E + e];
-        double dj = trace<ND>(sr);
-        sum += dj * s.volume[e];
-    }
-    s.ntmp[n] = sum / s.volume_n[n];
+        v[0] = trace<ND>(sr) * s.volume[e];
+    });
+    s.ntmp[n] = sum[0] / s.volume_n[n];
 }
 
 // compute_edvoldt (geometry.cxx:158-179)
+template <int ND> __device__ __forceinline__ double edvoldt_elem(const DevState &s, int e, const int *c)
+{
+    double dj = 0;
+#pragma unroll
+    for (int i = 0; i < Dim<ND>::NPE; ++i) dj += s.ntmp[c[i]];
+    return s.edvoldt[e] = dj / Dim<ND>::NPE;
+}
+
 template <int ND> __global__ __launch_bounds__(BLOCK) void k_edvoldt(DevState s)
 {
     BIND_ELEM(s, e);
     int c[Dim<ND>::NPE];
     load_conn<ND>(s, e, c);
-    double dj = 0;
-#pragma unroll
-    for (int i = 0; i < Dim<ND>::NPE; ++i) dj += s.ntmp[c[i]];
-    s.edvoldt[e] = dj / Dim<ND>::NPE;
+    edvoldt_elem<ND>(s, e, c);
 }
 
 // Non-temporal variants for arrays a pass streams once per step and no pass
@@ -407,21 +460,19 @@ __device__ __forceinline__ void set_error(DevScalars *sc, int code)
     atomicCAS(&sc->err, 0, code);
 }
 
-// update_stress (rheology.cxx:510-646)
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_update_stress(DevState s)
+// update_stress (rheology.cxx:510-646); returns the pressure change
+template <int ND> __device__ __forceinline__ double stress_elem(const DevState &s, int e, const int *c, double edvoldt,
+                                                              double vol)
 {
-    BIND_ELEM(s, e);
-    constexpr int NPE = Dim<ND>::NPE, NSTR = Dim<ND>::NSTR;
+    constexpr int NSTR = Dim<ND>::NSTR;
     const long E = s.E;
-    int c[NPE];
-    load_conn<ND>(s, e, c);
     double st[NSTR], es[NSTR], edot[NSTR];
     load_tensor<ND>(s.stress, E, e, st);
     load_tensor<ND>(s.strain, E, e, es);
     load_tensor<ND>(s.strain_rate, E, e, edot);
     double syy = s.stressyy[e], pl = s.plstrain[e], dpl = s.delta_plstrain[e], dp;
     double Tm = elem_mean<ND>(s.T, c);
-    bool ok = stress_update<ND>(s, e, s.sc->dt, s.edvoldt[e], Tm, s.volume[e], s.volume_old[e],
+    bool ok = stress_update<ND>(s, e, s.sc->dt, edvoldt, Tm, vol, s.volume_old[e],
                                 st, syy, es, edot, pl, dpl, dp);
     if (!ok) set_error(s.sc, DES_ERR_INPUT);
     store_tensor<ND>(s.stress, E, e, st);
@@ -431,19 +482,27 @@ template <int ND> __global__ __launch_bounds__(BLOCK) void k_update_stress(DevSt
     s.plstrain[e] = pl;
     s.delta_plstrain[e] = dpl;
     s.dpressure[e] = dp;
+    return dp;
+}
+
+template <int ND> __global__ __launch_bounds__(BLOCK) void k_update_stress(DevState s)
+{
+    BIND_ELEM(s, e);
+    int c[Dim<ND>::NPE];
+    load_conn<ND>(s, e, c);
+    stress_elem<ND>(s, e, c, s.edvoldt[e], s.volume[e]);
 }
 
 // NMD_stress (geometry.cxx:182-236): node average of dp into ntmp ...
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_nmd_node(DevState s)
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_nmd_node(DevState s)
 {
-    BIND_NODE(s, n);
-    constexpr int NPE = Dim<ND>::NPE;
-    double sum = 0;
-    for (int p = s.csr_off[n]; p < s.csr_off[n + 1]; ++p) {
-        int e = s.csr_ent[p] / NPE;
-        sum += s.dpressure[e] * s.volume[e];
-    }
-    s.ntmp[n] = sum / s.volume_n[n];
+    BIND_NODE_NB(s, n, NODE_BLOCK);
+    double sum[1];
+    list_sums(s, n, sum, [&](int ent, double *v) {
+        const int e = ent / Dim<ND>::NPE;
+        v[0] = s.dpressure[e] * s.volume[e];
+    });
+    s.ntmp[n] = sum[0] / s.volume_n[n];
 }
 
 // ... and the element correction of the stress diagonal
@@ -830,13 +889,13 @@ __device__ __forceinline__ void node_force(const DevState &s, int n, double f[ND
     }
 }
 
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_force_node(DevState s)
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_force_node(DevState s)
 {
-    BIND_NODE(s, n);
+    BIND_NODE_NB(s, n, NODE_BLOCK);
     double f[ND], v[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) v[d] = s.vel[d * s.N + n];
-    node_force<ND>(s, n, f, v);
+    node_force<ND, false, 8>(s, n, f, v);
 #pragma unroll
     for (int d = 0; d < ND; ++d) s.force[d * s.N + n] = f[d];
 }
@@ -1004,27 +1063,168 @@ template <int ND> __global__ __launch_bounds__(BLOCK) void k_update_coordinate(D
     for (int d = 0; d < ND; ++d) s.coord[d * s.N + n] += s.vel[d * s.N + n] * dt;
 }
 
-// rotate_stress (fields.cxx:411-483) with stored shape functions
-template <int ND> __global__ __launch_bounds__(BLOCK) void k_rotate(DevState s, int use_dt_prev)
+// rotate_stress (fields.cxx:411-483)
+template <int ND> __device__ __forceinline__ void rotate_elem(const DevState &s, int e, const int *c,
+                                                            const double sh[ND][Dim<ND>::NPE], double dt)
 {
-    BIND_ELEM(s, e);
-    // batched models close their steps in one launch: only the elastic ones
-    // rotate (dynearthsol.cxx:346-347)
-    if (s.eblk_model && !(s.P->rheol_type & DES_RH_ELASTIC)) return;
     constexpr int NPE = Dim<ND>::NPE, NSTR = Dim<ND>::NSTR;
-    int c[NPE];
-    load_conn<ND>(s, e, c);
-    double v[NPE][ND], sh[ND][NPE], w[3], st[NSTR], es[NSTR];
+    double v[NPE][ND], w[3], st[NSTR], es[NSTR];
     gather_vec<ND>(s.vel, s.N, c, v);
-    load_shp<ND>(s, e, sh);
     spin<ND>(v, sh, w);
-    const double dt = use_dt_prev ? s.sc->dt_prev : s.sc->dt;
     load_tensor<ND>(s.stress, s.E, e, st);
     load_tensor<ND>(s.strain, s.E, e, es);
     jaumann<ND>(st, dt, w);
     jaumann<ND>(es, dt, w);
     store_tensor<ND>(s.stress, s.E, e, st);
     store_tensor<ND>(s.strain, s.E, e, es);
+}
+
+template <int ND> __global__ __launch_bounds__(BLOCK) void k_rotate(DevState s)
+{
+    BIND_ELEM(s, e);
+    int c[Dim<ND>::NPE];
+    load_conn<ND>(s, e, c);
+    double sh[ND][Dim<ND>::NPE];
+    load_shp<ND>(s, e, sh);
+    rotate_elem<ND>(s, e, c, sh, s.sc->dt);
+}
+
+// ---- several reference functions in one launch
+//
+// Where one function's element (or node) reads only its own element's (or
+// node's) results of the one before, their kernels are one: a step through the
+// per-function kernels of a 100 k-tet model was 21 launches, most of them 3-5
+// us of launch and memory latency and no work (148 us a step); as 8 launches,
+// with the node sums above, it is 79 us.  Each array gets the value its own
+// kernel gives it.
+
+// volume, the element side of compute_mass, compute_shape_fn and, with rot,
+// rotate_stress of the step that ended (rot 1: by dt, 2: by dt_prev, which is
+// that step's dt once compute_dt has run)
+template <int ND> __global__ __launch_bounds__(BLOCK) void k_geometry(DevState s, int rot)
+{
+    BIND_ELEM(s, e);
+    constexpr int NPE = Dim<ND>::NPE;
+    int c[NPE];
+    load_conn<ND>(s, e, c);
+    double x[NPE][ND], sh[ND][NPE], m, tm;
+    gather_vec<ND>(s.coord, s.N, c, x);
+    const double vol = elem_volume<ND>(x);
+    s.volume[e] = vol;
+    mass_of<ND>(s, e, vol, elem_mean<ND>(s.T, c), m, tm);
+    mass_terms(s)[e] = make_double2(m, tm);
+    shape_fn<ND>(x, vol, sh);
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int i = 0; i < NPE; ++i) s.shp[(d * NPE + i) * (long)s.E + e] = sh[d][i];
+    // batched models close their steps in one launch: only the elastic ones
+    // rotate (dynearthsol.cxx:346-347)
+    if (!rot || (s.eblk_model && !(s.P->rheol_type & DES_RH_ELASTIC))) return;
+    rotate_elem<ND>(s, e, c, sh, rot == 2 ? s.sc->dt_prev : s.sc->dt);
+}
+
+// the start of a step (var.time, var.steps), the element side of
+// update_temperature, update_strain_rate, and the terms of compute_dvoldt
+template <int ND> __global__ __launch_bounds__(BLOCK) void k_step_rates(DevState s)
+{
+    BIND_ELEM(s, e);
+    if (e == 0) {
+        s.sc->time += s.sc->dt;
+        s.sc->steps += 1;
+    }
+    int c[Dim<ND>::NPE];
+    load_conn<ND>(s, e, c);
+    double sh[ND][Dim<ND>::NPE];
+    load_shp<ND>(s, e, sh);
+    if (s.P->has_thermal_diffusion) temp_elem<ND>(s, e, c, sh);
+    s.escal[e] = strain_rate_elem<ND>(s, e, c, sh) * s.volume[e];
+}
+
+// the node sides of update_temperature and compute_dvoldt
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_step_rates_node(DevState s)
+{
+    BIND_NODE_NB(s, n, NODE_BLOCK);
+    const bool thermal = s.P->has_thermal_diffusion;
+    const double vn = s.volume_n[n], T = s.T[n], tm = s.tmass[n];
+    double sum[2];
+    list_sums(s, n, sum, [&](int ent, double *v) {
+        v[0] = thermal ? s.ework[ent] : 0.0;
+        v[1] = s.escal[ent / Dim<ND>::NPE];
+    });
+    if (thermal) s.T[n] = temperature_new(s, n, T, sum[0], s.sc->dt, tm);
+    s.ntmp[n] = sum[1] / vn;
+}
+
+// compute_edvoldt, update_stress, and the terms of NMD_stress
+template <int ND> __global__ __launch_bounds__(BLOCK) void k_step_stress(DevState s)
+{
+    BIND_ELEM(s, e);
+    int c[Dim<ND>::NPE];
+    load_conn<ND>(s, e, c);
+    const double vol = s.volume[e];
+    s.escal[e] = stress_elem<ND>(s, e, c, edvoldt_elem<ND>(s, e, c), vol) * vol;
+}
+
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_step_nmd_node(DevState s)
+{
+    BIND_NODE_NB(s, n, NODE_BLOCK);
+    double sum[1];
+    list_sums(s, n, sum, [&](int ent, double *v) { v[0] = s.escal[ent / Dim<ND>::NPE]; });
+    s.ntmp[n] = sum[0] / s.volume_n[n];
+}
+
+// the element sides of NMD_stress and update_force on the first neb blocks,
+// the tractions of the loaded facets on the others
+template <int ND>
+__global__ __launch_bounds__(BLOCK) void k_step_force(DevState s, int neb, const int *facets, int nf)
+{
+    if ((int)blockIdx.x >= neb) {
+        const int t = (blockIdx.x - neb) * BLOCK + threadIdx.x;
+        if (t < nf) facet_traction_item<ND>(s, facets, t);
+        return;
+    }
+    BIND_ELEM_AT(s, e, xcd_block_of(neb, s.rev));
+    constexpr int NPE = Dim<ND>::NPE, NSTR = Dim<ND>::NSTR;
+    int c[NPE], pos[NPE];
+    load_conn<ND>(s, e, c);
+    double sh[ND][NPE], st[NSTR], out[NPE][ND];
+    load_shp<ND>(s, e, sh);
+    load_tensor<ND>(s.stress, s.E, e, st);
+    nmd_correct<ND>(s, e, c, st);
+#pragma unroll
+    for (int i = 0; i < ND; ++i) s.stress[i * (long)s.E + e] = st[i];
+    force_contrib<ND>(s, e, s.volume[e], sh, st, elem_mean<ND>(s.T, c), out);
+    force_slots<ND>(s, e, false, nullptr, pos);
+    store_force_contrib<ND>(s, pos, out);
+}
+
+// the node side of update_force, update_velocity, apply_vbcs and
+// update_mesh's coordinates
+template <int ND> __global__ __launch_bounds__(NODE_BLOCK) void k_step_move(DevState s)
+{
+    BIND_NODE_NB(s, n, NODE_BLOCK);
+    const double dt = s.sc->dt, m = s.mass[n];
+    const unsigned flag = s.bcflag[n];
+    double f[ND], v[ND], x[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        v[d] = s.vel[d * s.N + n];
+        x[d] = s.coord[d * s.N + n];
+    }
+    node_force<ND, false, 8>(s, n, f, v);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        s.force[d * s.N + n] = f[d];
+        v[d] += dt * f[d] / m;
+    }
+    if (flag & BOUND_ANY)
+        if (!vbc_node<ND>(s, flag, v)) set_error(s.sc, DES_ERR_ASSERT);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        s.vel[d * s.N + n] = v[d];
+        s.coord[d * s.N + n] = x[d] + v[d] * dt;
+    }
 }
 
 // ---- compute_dt (geometry.cxx:239-310): block minima, then one block
@@ -2270,13 +2470,6 @@ __global__ void k_clear_rotation(DevState s)
     s.sc->rot_pending = 0;
 }
 
-__global__ void k_step_begin(DevState s)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    s.sc->time += s.sc->dt;
-    s.sc->steps += 1;
-}
-
 // ---- the persistent launch: a whole run of fused steps in one kernel
 //
 // One cooperative launch holds as many workgroups as can be resident at once
@@ -2554,12 +2747,15 @@ int check_launch(des_ctx *ctx)
     return DES_OK;
 }
 
-#define LAUNCH_ND(kern, grid, ...)                                                        \
+#define LAUNCH_ND(kern, grid, ...) LAUNCH_NB(kern, grid, BLOCK, __VA_ARGS__)
+// a node kernel in blocks of NODE_BLOCK
+#define LAUNCH_NODE(kern, ...) LAUNCH_NB(kern, (ctx->N + NODE_BLOCK - 1) / NODE_BLOCK, NODE_BLOCK, __VA_ARGS__)
+#define LAUNCH_NB(kern, grid, nthreads, ...)                                                        \
     do {                                                                                  \
         if (ctx->nd == 3)                                                                 \
-            hipExtLaunchKernelGGL(kern<3>, dim3(grid), dim3(BLOCK), 0, ctx->stream, ctx->ev_a, ctx->ev_b, 0, __VA_ARGS__); \
+            hipExtLaunchKernelGGL(kern<3>, dim3(grid), dim3(nthreads), 0, ctx->stream, ctx->ev_a, ctx->ev_b, 0, __VA_ARGS__); \
         else                                                                              \
-            hipExtLaunchKernelGGL(kern<2>, dim3(grid), dim3(BLOCK), 0, ctx->stream, ctx->ev_a, ctx->ev_b, 0, __VA_ARGS__); \
+            hipExtLaunchKernelGGL(kern<2>, dim3(grid), dim3(nthreads), 0, ctx->stream, ctx->ev_a, ctx->ev_b, 0, __VA_ARGS__); \
         int rc_ = check_launch(ctx);                                                      \
         if (rc_) return rc_;                                                              \
     } while (0)
@@ -2577,23 +2773,55 @@ bool facet_loaded(const des_params &P, int i)
 // host AoS [n][k] <-> device SoA [k][stride], rows off .. off+n-1; device
 // row off + i holds host row perm[i] (i without perm)
 // Host-order AoS (row perm[i], k values per row) <-> device SoA (component j
-// of device row i at soa[j * stride + i]), one thread per device row
-__global__ __launch_bounds__(BLOCK) void k_soa_to_aos(const double *soa, long stride, long n, int k,
-                                                      const int *perm, double *aos)
+// of device row i at soa[j * stride + i]).  A block's rows pass through LDS, so
+// that K consecutive lanes touch one host row: the rows are scattered over the
+// host array (curve order), and a lane that writes its own row's values one by
+// one asks for every row's line K times (8.09 M stress tensors: 433 us, through
+// LDS 341 us).  K is k, the values per row (at most 6).
+template <int K, bool UP>
+__global__ __launch_bounds__(BLOCK) void k_rows(const double *src, double *dst, long stride, long n, const int *perm)
 {
-    const long i = blockIdx.x * (long)BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const long h = perm ? perm[i] : i;
-    for (int j = 0; j < k; ++j) aos[h * k + j] = soa[j * stride + i];
+    __shared__ double buf[BLOCK * K];
+    __shared__ int row[BLOCK];
+    const long i0 = blockIdx.x * (long)BLOCK, i = i0 + threadIdx.x;
+    const int nr = (int)min((long)BLOCK, n - i0);
+    if (perm) row[threadIdx.x] = i < n ? perm[i] : 0;
+    if constexpr (!UP) {
+        if (i < n)
+#pragma unroll
+            for (int j = 0; j < K; ++j) buf[threadIdx.x * K + j] = src[j * stride + i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int q = j * BLOCK + threadIdx.x, r = q / K;
+        if (r < nr) {
+            const long h = perm ? (long)row[r] : i0 + r;
+            if constexpr (UP) buf[q] = src[h * K + q % K];
+            else dst[h * K + q % K] = buf[q];
+        }
+    }
+    if constexpr (UP) {
+        __syncthreads();
+        if (i < n)
+#pragma unroll
+            for (int j = 0; j < K; ++j) dst[j * stride + i] = buf[threadIdx.x * K + j];
+    }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_aos_to_soa(const double *aos, long n, int k, const int *perm,
-                                                      double *soa, long stride)
+template <bool UP>
+void launch_rows(des_ctx *ctx, const double *src, double *dst, long stride, long n, int k, const int *perm)
 {
-    const long i = blockIdx.x * (long)BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const long h = perm ? perm[i] : i;
-    for (int j = 0; j < k; ++j) soa[j * stride + i] = aos[h * k + j];
+    const dim3 g(nblocks(n)), b(BLOCK);
+#define ROWS(K) hipLaunchKernelGGL((k_rows<K, UP>), g, b, 0, ctx->stream, src, dst, stride, n, perm)
+    switch (k) {
+    case 1: ROWS(1); break;
+    case 2: ROWS(2); break;
+    case 3: ROWS(3); break;
+    case 4: ROWS(4); break;
+    default: ROWS(6); break;       // 3D tensors
+    }
+#undef ROWS
 }
 
 // the device copy of a host permutation (a range of eh or nh)
@@ -2623,7 +2851,8 @@ int ensure_xfer(des_ctx *ctx, size_t n)
 
 // Transfers in the host's numbering: the rows are permuted and interleaved
 // on the device, and one copy crosses PCIe.
-// src_dev: src is device memory (host row order, AoS) and is read in place
+// src_dev: src is device memory (host row order, AoS) and is read in place, in
+// stream order: the caller synchronizes once after its last transfer
 int upload_soa(des_ctx *ctx, double *dst, const double *src, long n, int k, long stride = -1, long off = 0,
                const int *perm = nullptr, bool src_dev = false)
 {
@@ -2638,14 +2867,14 @@ int upload_soa(des_ctx *ctx, double *dst, const double *src, long n, int k, long
         HIPCHK(hipMemcpyAsync(ctx->xfer, src, sizeof(double) * n * k, hipMemcpyHostToDevice, ctx->stream));
         aos = ctx->xfer;
     }
-    hipLaunchKernelGGL(k_aos_to_soa, dim3(nblocks(n)), dim3(BLOCK), 0, ctx->stream, aos, n, k, dp,
-                       dst + off, stride);
+    launch_rows<true>(ctx, aos, dst + off, stride, n, k, dp);
     if ((rc = check_launch(ctx))) return rc;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (!src_dev) HIPCHK(hipStreamSynchronize(ctx->stream));
     return DES_OK;
 }
 
-// dst_dev: dst is device memory (host row order, AoS) written in place
+// dst_dev: dst is device memory (host row order, AoS) written in place, in
+// stream order as above
 int download_soa(des_ctx *ctx, double *dst, const double *src, long n, int k, long stride = -1, long off = 0,
                  const int *perm = nullptr, bool dst_dev = false)
 {
@@ -2655,11 +2884,10 @@ int download_soa(des_ctx *ctx, double *dst, const double *src, long n, int k, lo
     if (perm && !dp) return fail(ctx, DES_ERR_INPUT, "download: unknown row order");
     int rc;
     if (!dst_dev && (rc = ensure_xfer(ctx, (size_t)n * k))) return rc;
-    hipLaunchKernelGGL(k_soa_to_aos, dim3(nblocks(n)), dim3(BLOCK), 0, ctx->stream, src + off, stride, n, k, dp,
-                       dst_dev ? dst : ctx->xfer);
+    launch_rows<false>(ctx, src + off, dst_dev ? dst : ctx->xfer, stride, n, k, dp);
     if ((rc = check_launch(ctx))) return rc;
-    if (!dst_dev)
-        HIPCHK(hipMemcpyAsync(dst, ctx->xfer, sizeof(double) * n * k, hipMemcpyDeviceToHost, ctx->stream));
+    if (dst_dev) return DES_OK;
+    HIPCHK(hipMemcpyAsync(dst, ctx->xfer, sizeof(double) * n * k, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return DES_OK;
 }
@@ -2693,7 +2921,15 @@ int launch_compute_dt(des_ctx *ctx)
 int launch_mass(des_ctx *ctx)
 {
     LAUNCH_ND(k_mass_elem, nblocks(ctx->E), ctx->s);
-    LAUNCH_ND(k_mass_node, nblocks(ctx->N), ctx->s);
+    LAUNCH_NODE(k_mass_node, ctx->s);
+    return DES_OK;
+}
+
+// volume, mass, shape functions and, with rot, the Jaumann rotation (k_geometry)
+int launch_geometry(des_ctx *ctx, int rot)
+{
+    LAUNCH_ND(k_geometry, nblocks(ctx->E), ctx->s, rot);
+    LAUNCH_NODE(k_mass_node, ctx->s);
     return DES_OK;
 }
 
@@ -2701,18 +2937,14 @@ int launch_update_mesh(des_ctx *ctx)
 {
     LAUNCH_ND(k_update_coordinate, nblocks(ctx->N), ctx->s);
     swap_volume(ctx);
-    LAUNCH_ND(k_volume, nblocks(ctx->E), ctx->s);
-    int rc = launch_mass(ctx);
-    if (rc) return rc;
-    LAUNCH_ND(k_shape_fn, nblocks(ctx->E), ctx->s);
-    return DES_OK;
+    return launch_geometry(ctx, 0);
 }
 
 int launch_force(des_ctx *ctx)
 {
     LAUNCH_ND(k_force_elem, nblocks(ctx->E), ctx->s);
     if (ctx->nactive) LAUNCH_ND(k_facet_traction, nblocks(ctx->nactive), ctx->s, ctx->active_facets, ctx->nactive);
-    LAUNCH_ND(k_force_node, nblocks(ctx->N), ctx->s);
+    LAUNCH_NODE(k_force_node, ctx->s);
     return DES_OK;
 }
 
@@ -2723,17 +2955,12 @@ int flush_deferred(des_ctx *ctx)
     // the tail of the last step: update_mesh after update_coordinate, then
     // rotate_stress with that step's dt (dynearthsol.cxx:226-231, 346-347)
     swap_volume(ctx);
-    LAUNCH_ND(k_volume, nblocks(ctx->E), ctx->s);
-    int rc = launch_mass(ctx);
+    const int rc = launch_geometry(ctx, ctx->nmodels || (ctx->P.rheol_type & DES_RH_ELASTIC) ? 2 : 0);
     if (rc) return rc;
-    LAUNCH_ND(k_shape_fn, nblocks(ctx->E), ctx->s);
-    if (ctx->nmodels) {          // k_rotate skips the models without elasticity
-        LAUNCH_ND(k_rotate, nblocks(ctx->E), ctx->s, 1);
+    if (ctx->nmodels)
         hipLaunchKernelGGL(k_clear_rotation_b, dim3(nblocks(ctx->nmodels)), dim3(BLOCK), 0, ctx->stream, ctx->s);
-    } else {
-        if (ctx->P.rheol_type & DES_RH_ELASTIC) LAUNCH_ND(k_rotate, nblocks(ctx->E), ctx->s, 1);
+    else
         hipLaunchKernelGGL(k_clear_rotation, dim3(1), dim3(1), 0, ctx->stream, ctx->s);
-    }
     ctx->closing_pending = false;
     return check_launch(ctx);
 }
@@ -3384,8 +3611,8 @@ int xfer_fields(des_ctx *ctx, des_fields *f, bool up, int model, bool dev = fals
             if (f->elem_visc) ctx->has_visc[model] = 1;
             if (f->elem_cohesion) ctx->has_coh[model] = 1;
         }
-        HIPCHK(hipStreamSynchronize(ctx->stream));
     }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
     return DES_OK;
 }
 
@@ -3719,28 +3946,26 @@ ENTRY(des_compute_volume, LAUNCH_ND(k_volume, nblocks(ctx->E), ctx->s))
 ENTRY(des_compute_mass, if ((rc = launch_mass(ctx))) return rc)
 ENTRY(des_compute_shape_fn, LAUNCH_ND(k_shape_fn, nblocks(ctx->E), ctx->s))
 ENTRY(des_update_temperature, LAUNCH_ND(k_temp_elem, nblocks(ctx->E), ctx->s);
-      LAUNCH_ND(k_temp_node, nblocks(ctx->N), ctx->s))
+      LAUNCH_NODE(k_temp_node, ctx->s))
 ENTRY(des_update_strain_rate, LAUNCH_ND(k_strain_rate, nblocks(ctx->E), ctx->s))
-ENTRY(des_compute_dvoldt, LAUNCH_ND(k_dvoldt_node, nblocks(ctx->N), ctx->s))
+ENTRY(des_compute_dvoldt, LAUNCH_NODE(k_dvoldt_node, ctx->s))
 ENTRY(des_compute_edvoldt, LAUNCH_ND(k_edvoldt, nblocks(ctx->E), ctx->s))
 ENTRY(des_update_stress, LAUNCH_ND(k_update_stress, nblocks(ctx->E), ctx->s))
-ENTRY(des_nmd_stress, LAUNCH_ND(k_nmd_node, nblocks(ctx->N), ctx->s);
+ENTRY(des_nmd_stress, LAUNCH_NODE(k_nmd_node, ctx->s);
       LAUNCH_ND(k_nmd_elem, nblocks(ctx->E), ctx->s))
 ENTRY(des_update_force, if ((rc = launch_force(ctx))) return rc)
 ENTRY(des_update_velocity, LAUNCH_ND(k_update_velocity, nblocks(ctx->N), ctx->s))
 ENTRY(des_apply_vbcs, LAUNCH_ND(k_apply_vbcs, nblocks(ctx->N), ctx->s))
 ENTRY(des_update_mesh, if ((rc = launch_update_mesh(ctx))) return rc)
-ENTRY(des_rotate_stress, LAUNCH_ND(k_rotate, nblocks(ctx->E), ctx->s, 0))
+ENTRY(des_rotate_stress, LAUNCH_ND(k_rotate, nblocks(ctx->E), ctx->s))
 
 int des_init_derived(des_ctx *ctx)
 {
     if (!ctx) return DES_ERR_INPUT;
     int rc = flush_deferred(ctx);
     if (rc) return rc;
-    LAUNCH_ND(k_volume, nblocks(ctx->E), ctx->s);
+    if ((rc = launch_geometry(ctx, 0))) return rc;
     HIPCHK(hipMemcpyAsync(ctx->s.volume_old, ctx->s.volume, sizeof(double) * ctx->E, hipMemcpyDeviceToDevice, ctx->stream));
-    if ((rc = launch_mass(ctx))) return rc;
-    LAUNCH_ND(k_shape_fn, nblocks(ctx->E), ctx->s);
     return DES_OK;
 }
 
@@ -3917,24 +4142,16 @@ int des_step(des_ctx *ctx)
     if (!ctx) return DES_ERR_INPUT;
     int rc = flush_deferred(ctx);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, ctx->stream, ctx->s);
-    if ((rc = check_launch(ctx))) return rc;
     ctx->steps++;
-    if (ctx->P.has_thermal_diffusion) {
-        LAUNCH_ND(k_temp_elem, nblocks(ctx->E), ctx->s);
-        LAUNCH_ND(k_temp_node, nblocks(ctx->N), ctx->s);
-    }
-    LAUNCH_ND(k_strain_rate, nblocks(ctx->E), ctx->s);
-    LAUNCH_ND(k_dvoldt_node, nblocks(ctx->N), ctx->s);
-    LAUNCH_ND(k_edvoldt, nblocks(ctx->E), ctx->s);
-    LAUNCH_ND(k_update_stress, nblocks(ctx->E), ctx->s);
-    LAUNCH_ND(k_nmd_node, nblocks(ctx->N), ctx->s);
-    LAUNCH_ND(k_nmd_elem, nblocks(ctx->E), ctx->s);
-    if ((rc = launch_force(ctx))) return rc;
-    LAUNCH_ND(k_update_velocity, nblocks(ctx->N), ctx->s);
-    LAUNCH_ND(k_apply_vbcs, nblocks(ctx->N), ctx->s);
-    if ((rc = launch_update_mesh(ctx))) return rc;
-    if (ctx->P.rheol_type & DES_RH_ELASTIC) LAUNCH_ND(k_rotate, nblocks(ctx->E), ctx->s, 0);
+    LAUNCH_ND(k_step_rates, nblocks(ctx->E), ctx->s);
+    LAUNCH_NODE(k_step_rates_node, ctx->s);
+    LAUNCH_ND(k_step_stress, nblocks(ctx->E), ctx->s);
+    LAUNCH_NODE(k_step_nmd_node, ctx->s);
+    const int neb = nblocks(ctx->E);
+    LAUNCH_ND(k_step_force, neb + nblocks(ctx->nactive), ctx->s, neb, ctx->active_facets, ctx->nactive);
+    LAUNCH_NODE(k_step_move, ctx->s);
+    swap_volume(ctx);
+    if ((rc = launch_geometry(ctx, ctx->P.rheol_type & DES_RH_ELASTIC ? 1 : 0))) return rc;
     if (ctx->steps % 10 == 0)
         if ((rc = launch_compute_dt(ctx))) return rc;
     return DES_OK;
