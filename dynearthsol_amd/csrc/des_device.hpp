@@ -83,6 +83,8 @@ struct DevState {
     const int *slot;                              // E x NPE: CSR position of entry e*NPE+i
     const unsigned *srank;                        // E: byte i = position of entry e*NPE+i in its
                                                   // node's list (null: a list longer than 256)
+    const unsigned *wrank;                        // E: byte i = rank of entry e*NPE+i's position
+                                                  // among those of e's wave (k_wave_ranks)
     double *erec;                                 // E x 8 packed records (fused pass A -> B)
     double *escal;                                // 4 x E element scalars
     double *ftrac;                                // nbf x ND facet tractions
