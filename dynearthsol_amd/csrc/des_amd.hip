@@ -2033,15 +2033,15 @@ __device__ __forceinline__ void pass_c_ret_item(const DevState &s, int k)
         const double bulkm = harmonic_mean(st, P->bulk_modulus, e);
         const double shearm = harmonic_mean(st, P->shear_modulus, e);
         const double pl = s.plstrain[e];
+        // requested before the return, which is a chain of some thousand
+        // operations that its loads would only lengthen
+        double sv[6];
+        const bool evp = P->rheol_type == DES_RH_EVP;
+        if (evp) load_tensor<3>(s.stress, s.E, e, sv);
         double amc, anphi, anpsi, hardn, ten_max, depls;
         mat_plastic_props(st, e, pl, amc, anphi, anpsi, hardn, ten_max);
         mc_return<3>(bulkm, shearm, amc, anphi, anpsi, hardn, ten_max, depls, sp);
-        bool take = true;
-        if (P->rheol_type == DES_RH_EVP) {
-            double sv[6];
-            load_tensor<3>(s.stress, s.E, e, sv);
-            take = !(second_invariant2<3>(sv) < second_invariant2<3>(sp));
-        }
+        const bool take = !(evp && second_invariant2<3>(sv) < second_invariant2<3>(sp));
         if (take) {
             store_tensor<3>(s.stress, s.E, e, sp);
             s.plstrain[e] = pl + depls;
@@ -4587,13 +4587,16 @@ bool any_plastic(const des_ctx *ctx)
     return false;
 }
 
-// the Mohr-Coulomb returns that pass C deferred (3D): wavefronts of 64 lanes,
-// each for at least four list segments (256 elements) and at most 2048 of
-// them, what the chip holds of this kernel at its register count
+// the Mohr-Coulomb returns that pass C deferred (3D): a wavefront per list
+// segment (64 elements), at most 2048 of them, what the chip holds of this
+// kernel at its register count.  A return is a long chain and a wavefront runs
+// every lane's branches of the eigen solve: a sixth of 200 k tets listed took
+// 28.4 us in 782 wavefronts with 43 returns each, 20.8 in 2048 with 16, and
+// 21.3 in 3125, which are more than fit at once.
 int launch_pass_c_ret(des_ctx *ctx, bool mixed = false)
 {
     if (ctx->nd != 3 || !any_plastic(ctx)) return DES_OK;
-    const dim3 g(std::min(nblocks(ctx->E), 2048)), b(64);
+    const dim3 g(std::min((ctx->E + 63) / 64, 2048)), b(64);
     if (mixed) hipExtLaunchKernelGGL(k_pass_c_ret_mixed, g, b, 0, ctx->stream, ctx->ev_a, ctx->ev_b, 0, ctx->s);
     else hipExtLaunchKernelGGL(k_pass_c_ret, g, b, 0, ctx->stream, ctx->ev_a, ctx->ev_b, 0, ctx->s);
     return check_launch(ctx);
