@@ -1618,6 +1618,7 @@ struct FusedFlags {
     int use_stored_mass = 0;   // first step after a sync: mass/tmass/volume_n from compute_mass
     int store_aux = 0;         // last step before a sync: keep strain_rate, edvoldt, force
     int step_end = 0;          // pass F also ends the step: time, steps, dt_prev, rotation flag
+    int slot_order = 0;        // pass E's full waves store their contributions in slot order
     // the differentiated run's step records, written by the pass that has
     // the value at hand (null in plain runs): pass C (FP64) the stress,
     // plastic strain and volume_old it starts from, pass B the node records
@@ -2180,7 +2181,7 @@ template <int ND, bool STAGE, int WPE = 1> __global__ __launch_bounds__(BLOCK, W
         pli[2] = s.wrank[e0];
     }
     const bool staged = STAGE && stage_block(s, blk, lds.stage, loff);
-    pass_e_body<ND>(s, fl, blk, staged, lds.stage, loff, lds.slots + threadIdx.x / 64, STAGE ? pre : nullptr,
+    pass_e_body<ND>(s, fl, blk, staged, lds.stage, loff, fl.slot_order ? lds.slots + threadIdx.x / 64 : nullptr, STAGE ? pre : nullptr,
                     STAGE ? pli : nullptr);
 }
 
@@ -2543,7 +2544,7 @@ template <int ND, bool STAGE> __global__ __launch_bounds__(BLOCK) void k_pass_e_
     }
     const bool staged = STAGE && stage_block(s, blk, lds.stage, loff);
     pass_e_mixed_body<ND>(s, fl, blk, staged, lds.stage, STAGE ? pre : nullptr, STAGE ? psd : nullptr,
-                          STAGE ? pli : nullptr, loff, lds.slots + threadIdx.x / 64);
+                          STAGE ? pli : nullptr, loff, fl.slot_order ? lds.slots + threadIdx.x / 64 : nullptr);
 }
 
 // node records from the SoA state, at the start of a fused run
@@ -4498,8 +4499,17 @@ int launch_pass_d(des_ctx *ctx, const FusedFlags &fl, int variant)
     return DES_OK;
 }
 
-int launch_pass_e(des_ctx *ctx, const FusedFlags &fl, bool mixed, int variant)
+// Pass E's stores in slot order cost a wave a trip through LDS, and pay where
+// the stores of many waves queue for the L2: 3D from 200 k elements on (16.5 ->
+// 13.0 us there).  With fewer blocks than the chip has CUs each wave has the
+// memory to itself and the trip is what is left: 100 steps of 3,948 triangles
+// took 3.35 ms with it and 3.14 without.
+constexpr int SLOT_ORDER_MIN = 256 * BLOCK;
+
+int launch_pass_e(des_ctx *ctx, const FusedFlags &fl0, bool mixed, int variant)
 {
+    FusedFlags fl = fl0;
+    fl.slot_order = ctx->E >= SLOT_ORDER_MIN;
     if (mixed) {
         if (variant == 1) LAUNCH_T2(k_pass_e_mixed, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
         else LAUNCH_T2(k_pass_e_mixed, true, BLOCK, nblocks(ctx->E), ctx->s, fl);

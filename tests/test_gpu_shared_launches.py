@@ -36,9 +36,11 @@ def test_step_equals_its_functions_one_by_one(name):
     _same(g.download(), h.download())
 
 
-# element counts whose last block ends in a full wave, a part of one or a single element
-@pytest.mark.parametrize("name,nelem", [("evp3", 300), ("evp3", 900), ("mat3", 1500), ("evp3", 2400), ("evp2", 250),
-                                        ("mat2", 700), ("maxwell2", 1300)])
+# above 65,536 elements the waves store (batches count all their models), below
+# it the lanes; the last block of each model ends in a full wave or in a part
+# of one
+@pytest.mark.parametrize("name,nelem", [("evp3", 900), ("evp2", 700), ("evp3", 66000), ("mat3", 70000), ("evp2", 66000),
+                                        ("mat2", 68000), ("maxwell3", 68500)])
 @pytest.mark.parametrize("mixed", [False, True])
 def test_force_slots_stored_by_waves_and_by_lanes(name, nelem, mixed):
     from dynearthsol_amd.lib import DesModel
@@ -52,3 +54,19 @@ def test_force_slots_stored_by_waves_and_by_lanes(name, nelem, mixed):
         out.append(g.download())
         g.close()
     _same(*out)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_force_slots_of_a_batch_with_part_blocks(mixed):
+    from dynearthsol_amd.lib import DesBatch
+    models = [SC.build("evp3", nelem=n) for n in (66000, 300, 900, 1500)]
+    print([m.nelem % 256 for m in models], "in the last blocks", flush=True)
+    out = []
+    for mode in (0, 1):
+        b = DesBatch(models)
+        b.set_launch_mode(mode)
+        b.run(8, abi.DES_MIXED if mixed else abi.DES_FP64)
+        out.append([b.download(k) for k in range(len(models))])
+        b.close()
+    for a, c in zip(*out):
+        _same(a, c)
