@@ -2,8 +2,9 @@
 // the DynEarthSol explicit time step.
 //
 // Two ways through a step:
-//   * per-function kernels, one per reference function, in the order of the
-//     reference's main loop (des_step, dynearthsol.cxx:325-361);
+//   * per-function kernels, one per reference function (the entry points), and
+//     the same functions sharing eight launches in the order of the reference's
+//     main loop (des_step, dynearthsol.cxx:325-361);
 //   * the fused six-pass schedule (des_run): three element passes and three
 //     node passes per step, shape functions and strain rates recomputed in
 //     registers instead of stored, mass / volume_n / tmass built inside the
