@@ -2961,7 +2961,8 @@ int ensure_xfer(des_ctx *ctx, size_t n)
 // Transfers in the host's numbering: the rows are permuted and interleaved
 // on the device, and one copy crosses PCIe.
 // src_dev: src is device memory (host row order, AoS) and is read in place, in
-// stream order: the caller synchronizes once after its last transfer
+// stream order: the caller waits for the stream before it returns, also when a
+// later call fails (wait_returning)
 int upload_soa(des_ctx *ctx, double *dst, const double *src, long n, int k, long stride = -1, long off = 0,
                const int *perm = nullptr, bool src_dev = false)
 {
@@ -3680,10 +3681,21 @@ int field_opt(des_ctx *ctx, double **slot, const double *src, long n, long off, 
     return upload_soa(ctx, *slot, src, n, 1, ctx->E, off, ctx->eh.data() + off, dev);
 }
 
+// Waits for the context's stream with the status of a call whose kernels use
+// the caller's device memory: also a call that failed half way leaves none of
+// them running when it returns.
+int wait_returning(des_ctx *ctx, int rc)
+{
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (rc || e == hipSuccess) return rc;
+    return fail(ctx, DES_ERR_HIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(e));
+}
+
 // The fields of des_fields between AoS arrays in host row order and the
 // device SoA state: the whole context (model < 0) or batched model `model` of
-// a group.  dev: the des_fields pointers are device memory.
-int xfer_fields(des_ctx *ctx, des_fields *f, bool up, int model, bool dev = false)
+// a group.  dev: the des_fields pointers are device memory.  Queues the work;
+// xfer_fields waits for it.
+int queue_fields(des_ctx *ctx, des_fields *f, bool up, int model, bool dev)
 {
     int rc = flush_deferred(ctx);
     if (rc) return rc;
@@ -3730,8 +3742,12 @@ int xfer_fields(des_ctx *ctx, des_fields *f, bool up, int model, bool dev = fals
             if (f->elem_cohesion) ctx->has_coh[model] = 1;
         }
     }
-    HIPCHK(hipStreamSynchronize(ctx->stream));
     return DES_OK;
+}
+
+int xfer_fields(des_ctx *ctx, des_fields *f, bool up, int model, bool dev = false)
+{
+    return wait_returning(ctx, queue_fields(ctx, f, up, model, dev));
 }
 
 }  // namespace
