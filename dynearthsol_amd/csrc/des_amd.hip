@@ -2153,7 +2153,7 @@ __device__ __forceinline__ void pass_e_body(DevState s, const FusedFlags &fl, in
     }
 }
 
-template <int ND, bool STAGE, int WPE = 1> __global__ __launch_bounds__(BLOCK, WPE) void k_pass_e(DevState s, FusedFlags fl)
+template <int ND, bool STAGE> __global__ __launch_bounds__(BLOCK) void k_pass_e(DevState s, FusedFlags fl)
 {
     // the contributions' LDS takes the place of the staged records
     union Lds {
@@ -4533,9 +4533,12 @@ int launch_pass_e(des_ctx *ctx, const FusedFlags &fl0, bool mixed, int variant)
     } else if (g_force_layout == 1) {
         if (variant == 1) LAUNCH_T2(k_pass_e_er, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
         else LAUNCH_T2(k_pass_e_er, true, BLOCK, nblocks(ctx->E), ctx->s, fl);
-    } else {     // staged (0), direct (1), staged with at least 8 waves per SIMD (2)
-        if (variant == 2) LAUNCH_E3(k_pass_e, true, 8, nblocks(ctx->E), ctx->s, fl);
-        else if (variant == 1) LAUNCH_T2(k_pass_e, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
+    } else {
+        // direct (1) or staged (0, and 2: a bound to 8 waves per SIMD, which
+        // the 29,696 bytes of LDS of 3D blocks do not allow -- 5 blocks a CU --
+        // and which without slot order spilled and took 62 us against 47 at
+        // 1.02 M tets)
+        if (variant == 1) LAUNCH_T2(k_pass_e, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
         else LAUNCH_T2(k_pass_e, true, BLOCK, nblocks(ctx->E), ctx->s, fl);
     }
     return DES_OK;
