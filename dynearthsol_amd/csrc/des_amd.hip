@@ -184,8 +184,8 @@ template <int ND> __device__ __forceinline__ void bind_model(DevState &s, int m)
 // Sums over node n's list in its (ascending host element) order: load(entry, v)
 // gives the K terms of an entry.  DEPTH entries are requested together and the
 // last, ragged round like the others (its missing entries repeat the last one
-// and are not added), so a list of 24 costs three round trips to memory.  One
-// entry at a time, in blocks of 256 threads, the node sums of a 100 k-tet model
+// and are not added), so a list of 24 costs three rounds of two dependent loads
+// (the entries, then their terms).  One entry at a time, in blocks of 256 threads, the node sums of a 100 k-tet model
 // took 12-16 us each; eight at a time in blocks of 64 (one wavefront per CU at
 // that size) 5.5-7 us, and k_mass_node of 8.09 M tets 1034 -> 234 us.
 constexpr int NODE_BLOCK = 64;
@@ -1163,9 +1163,9 @@ template <int ND> __global__ __launch_bounds__(BLOCK) void k_rotate(DevState s)
 //
 // Where one function's element (or node) reads only its own element's (or
 // node's) results of the one before, their kernels are one: a step through the
-// per-function kernels of a 100 k-tet model was 21 launches, most of them 3-5
-// us of launch and memory latency and no work (148 us a step); as 8 launches,
-// with the node sums above, it is 79 us.  Each array gets the value its own
+// per-function kernels of a 100 k-tet model was 20 launches (compute_dt every
+// tenth step aside), most of them 3-5 us of launch and memory latency and no
+// work (148 us a step); as 8 launches, with the node sums above, it is 79 us.  Each array gets the value its own
 // kernel gives it.
 
 // volume, the element side of compute_mass, compute_shape_fn and, with rot,
@@ -1992,8 +1992,8 @@ __device__ __forceinline__ void pass_c_blk(DevState s, const FusedFlags &fl, int
 
 // PLASTIC_ONLY: the instantiation for 3D contexts whose models are all
 // elasto-(visco-)plastic, without the other rheologies' code (whose registers
-// would otherwise set the kernel's allocation: 119 VGPRs direct and 107 staged
-// instead of 131 and 133, four waves per SIMD instead of three)
+// would otherwise set the kernel's allocation: 119 VGPRs direct instead of 131,
+// four waves per SIMD instead of three; staged both hold 123, four waves)
 template <int ND, int WPE, bool STAGE, bool PLASTIC_ONLY = false>
 __global__ __launch_bounds__(BLOCK, WPE) void k_pass_c(DevState s, FusedFlags fl)
 {
@@ -4517,10 +4517,18 @@ int launch_pass_d(des_ctx *ctx, const FusedFlags &fl, int variant)
 }
 
 // Pass E's stores in slot order cost a wave a trip through LDS, and pay where
-// the stores of many waves queue for the L2: 3D from 200 k elements on (16.5 ->
-// 13.0 us there).  With fewer blocks than the chip has CUs each wave has the
-// memory to itself and the trip is what is left: 100 steps of 3,948 triangles
-// took 3.35 ms with it and 3.14 without.
+// the stores of many waves queue for the L2: from about a block per CU on.  us
+// a launch, lanes' own stores -> slot order, staged (direct):
+//                    FP64                           mixed
+//   4 k triangles     4.9 ->  5.0 ( 4.1 ->  4.5)     4.6 ->  4.8 ( 4.1 ->  4.5)
+//   70 k              5.8 ->  5.8 ( 5.3 ->  5.1)     5.5 ->  5.5 ( 4.6 ->  4.8)
+//   250 k             9.9 ->  9.4 ( 9.1 ->  8.4)     7.5 ->  7.1 ( 6.8 ->  6.8)
+//   12 k tets         5.9 ->  5.4 ( 5.4 ->  5.3)     4.8 ->  5.1 ( 4.6 ->  5.5)
+//   50 k              7.0 ->  6.3 ( 6.9 ->  6.2)     5.2 ->  5.3 ( 5.3 ->  5.5)
+//   70 k              8.6 ->  7.0 ( 8.8 ->  7.6)     6.5 ->  6.4 ( 6.8 ->  6.9)
+//   200 k            14.4 -> 11.4 (15.4 -> 12.0)     9.6 ->  9.1 (10.3 -> 10.1)
+// A difference of 0.3 us is within what one side's launches vary by: from
+// 65,536 elements on nothing is slower, below it only 3D FP64 would gain.
 constexpr int SLOT_ORDER_MIN = 256 * BLOCK;
 
 int launch_pass_e(des_ctx *ctx, const FusedFlags &fl0, bool mixed, int variant)
@@ -4622,7 +4630,10 @@ bool any_plastic(const des_ctx *ctx)
 // kernel at its register count.  A return is a long chain and a wavefront runs
 // every lane's branches of the eigen solve: a sixth of 200 k tets listed took
 // 28.4 us in 782 wavefronts with 43 returns each, 20.8 in 2048 with 16, and
-// 21.3 in 3125, which are more than fit at once.
+// 21.3 in 3125, which are more than fit at once.  The mixed kernel (187 VGPRs,
+// two waves per SIMD too) takes 20.4 us there and 85 at 1.02 M tets, where one
+// list for all and QL out of line took 34 and 138; held to three waves by a
+// bound, in 3072 wavefronts, it spills and takes 22.3 and 82.
 int launch_pass_c_ret(des_ctx *ctx, bool mixed = false)
 {
     if (ctx->nd != 3 || !any_plastic(ctx)) return DES_OK;
