@@ -1619,7 +1619,6 @@ struct FusedFlags {
     int use_stored_mass = 0;   // first step after a sync: mass/tmass/volume_n from compute_mass
     int store_aux = 0;         // last step before a sync: keep strain_rate, edvoldt, force
     int step_end = 0;          // pass F also ends the step: time, steps, dt_prev, rotation flag
-    int slot_order = 0;        // pass E's full waves store their contributions in slot order
     // the differentiated run's step records, written by the pass that has
     // the value at hand (null in plain runs): pass C (FP64) the stress,
     // plastic strain and volume_old it starts from, pass B the node records
@@ -2161,12 +2160,17 @@ __device__ __forceinline__ void pass_e_body(DevState s, const FusedFlags &fl, in
     }
 }
 
-template <int ND, bool STAGE> __global__ __launch_bounds__(BLOCK) void k_pass_e(DevState s, FusedFlags fl)
+// SLOTS: full waves store their contributions in slot order.  A switch of the
+// kernel and not of its arguments: a small model's blocks are then free of the
+// LDS and the rank, 3D holds 72 instead of 76 VGPRs (7 waves per SIMD instead
+// of 5), and a step of 4 k triangles takes 30.1 us instead of 30.4, of 45 k
+// 33.7 instead of 34.0
+template <int ND, bool STAGE, bool SLOTS> __global__ __launch_bounds__(BLOCK) void k_pass_e(DevState s, FusedFlags fl)
 {
     // the contributions' LDS takes the place of the staged records
     union Lds {
         double2 stage[STAGE ? STAGE_MAX * (NREC / 2) : 1];
-        SlotBuf<ND, double> slots[BLOCK / 64];
+        SlotBuf<ND, double> slots[SLOTS ? BLOCK / 64 : 1];
     };
     __shared__ __align__(16) char mem[sizeof(Lds)];
     Lds &lds = *reinterpret_cast<Lds *>(mem);
@@ -2187,11 +2191,11 @@ template <int ND, bool STAGE> __global__ __launch_bounds__(BLOCK) void k_pass_e(
         pre[NSTR] = s.dpressure[e0];
         if (s.stage) pli[0] = s.stage_lidx[e0];
         if (s.srank) pli[1] = s.srank[e0];
-        pli[2] = s.wrank[e0];
+        if constexpr (SLOTS) pli[2] = s.wrank[e0];
     }
     const bool staged = STAGE && stage_block(s, blk, lds.stage, loff);
-    pass_e_body<ND>(s, fl, blk, staged, lds.stage, loff, fl.slot_order ? lds.slots + threadIdx.x / 64 : nullptr, STAGE ? pre : nullptr,
-                    STAGE ? pli : nullptr);
+    pass_e_body<ND>(s, fl, blk, staged, lds.stage, loff, SLOTS ? lds.slots + threadIdx.x / 64 : nullptr,
+                    STAGE ? pre : nullptr, STAGE ? pli : nullptr);
 }
 
 // pass E writing element-major force records
@@ -2523,11 +2527,12 @@ template <int ND> __device__ __forceinline__ void pass_e_mixed_body(DevState s, 
     if (valid) store_force_contrib_f32<ND>(s, pos, out);
 }
 
-template <int ND, bool STAGE> __global__ __launch_bounds__(BLOCK) void k_pass_e_mixed(DevState s, FusedFlags fl)
+template <int ND, bool STAGE, bool SLOTS>
+__global__ __launch_bounds__(BLOCK) void k_pass_e_mixed(DevState s, FusedFlags fl)
 {
     union Lds {
         double2 stage[STAGE ? STAGE_MAX * (NREC / 2) : 1];
-        SlotBuf<ND, float> slots[BLOCK / 64];
+        SlotBuf<ND, float> slots[SLOTS ? BLOCK / 64 : 1];
     };
     __shared__ __align__(16) char mem[sizeof(Lds)];
     Lds &lds = *reinterpret_cast<Lds *>(mem);
@@ -2549,11 +2554,11 @@ template <int ND, bool STAGE> __global__ __launch_bounds__(BLOCK) void k_pass_e_
         for (int k = 0; k < NSTR; ++k) psd[k] = s.sdev[k * (long)s.E + e0];
         if (s.stage) pli[0] = s.stage_lidx[e0];
         if (s.srank) pli[1] = s.srank[e0];
-        pli[2] = s.wrank[e0];
+        if constexpr (SLOTS) pli[2] = s.wrank[e0];
     }
     const bool staged = STAGE && stage_block(s, blk, lds.stage, loff);
     pass_e_mixed_body<ND>(s, fl, blk, staged, lds.stage, STAGE ? pre : nullptr, STAGE ? psd : nullptr,
-                          STAGE ? pli : nullptr, loff, fl.slot_order ? lds.slots + threadIdx.x / 64 : nullptr);
+                          STAGE ? pli : nullptr, loff, SLOTS ? lds.slots + threadIdx.x / 64 : nullptr);
 }
 
 // node records from the SoA state, at the start of a fused run
@@ -4544,25 +4549,32 @@ int launch_pass_d(des_ctx *ctx, const FusedFlags &fl, int variant)
 // 65,536 elements on nothing is slower, below it only 3D FP64 would gain.
 constexpr int SLOT_ORDER_MIN = 256 * BLOCK;
 
-int launch_pass_e(des_ctx *ctx, const FusedFlags &fl0, bool mixed, int variant)
+template <bool SLOTS> int launch_pass_e_slots(des_ctx *ctx, const FusedFlags &fl, bool mixed, int variant)
 {
-    FusedFlags fl = fl0;
-    fl.slot_order = ctx->E >= SLOT_ORDER_MIN;
+    const int g = nblocks(ctx->E);
     if (mixed) {
-        if (variant == 1) LAUNCH_T2(k_pass_e_mixed, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
-        else LAUNCH_T2(k_pass_e_mixed, true, BLOCK, nblocks(ctx->E), ctx->s, fl);
-    } else if (g_force_layout == 1) {
-        if (variant == 1) LAUNCH_T2(k_pass_e_er, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
-        else LAUNCH_T2(k_pass_e_er, true, BLOCK, nblocks(ctx->E), ctx->s, fl);
+        if (variant == 1) LAUNCH_E3(k_pass_e_mixed, false, SLOTS, g, ctx->s, fl);
+        else LAUNCH_E3(k_pass_e_mixed, true, SLOTS, g, ctx->s, fl);
     } else {
         // direct (1) or staged (0, and 2: a bound to 8 waves per SIMD, which
         // the 29,696 bytes of LDS of 3D blocks do not allow -- 5 blocks a CU --
         // and which without slot order spilled and took 62 us against 47 at
         // 1.02 M tets)
-        if (variant == 1) LAUNCH_T2(k_pass_e, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
-        else LAUNCH_T2(k_pass_e, true, BLOCK, nblocks(ctx->E), ctx->s, fl);
+        if (variant == 1) LAUNCH_E3(k_pass_e, false, SLOTS, g, ctx->s, fl);
+        else LAUNCH_E3(k_pass_e, true, SLOTS, g, ctx->s, fl);
     }
     return DES_OK;
+}
+
+int launch_pass_e(des_ctx *ctx, const FusedFlags &fl, bool mixed, int variant)
+{
+    if (!mixed && g_force_layout == 1) {
+        if (variant == 1) LAUNCH_T2(k_pass_e_er, false, BLOCK, nblocks(ctx->E), ctx->s, fl);
+        else LAUNCH_T2(k_pass_e_er, true, BLOCK, nblocks(ctx->E), ctx->s, fl);
+        return DES_OK;
+    }
+    return ctx->E >= SLOT_ORDER_MIN ? launch_pass_e_slots<true>(ctx, fl, mixed, variant)
+                                    : launch_pass_e_slots<false>(ctx, fl, mixed, variant);
 }
 
 int launch_pass_f(des_ctx *ctx, const FusedFlags &fl, bool mixed, int variant)
