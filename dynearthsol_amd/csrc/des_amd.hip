@@ -2701,9 +2701,11 @@ __global__ __launch_bounds__(BLOCK, 2) void k_persistent(const DevState *__restr
         grid.sync();
         if constexpr (HAS3) {
             if (g3.plastic) {       // the deferred Mohr-Coulomb returns (3D only)
-                const DevState s = pstate(ps3, k + pa.swap0);
-                const int w = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6), W = gridDim.x * (BLOCK / 64);
-                if (__hip_atomic_load(s.ret_any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                // the calls take the state in scratch: copied there only where
+                // there is a call (3D, 12 k tets: 4.0 -> 3.6 ms for 50 steps)
+                if (__hip_atomic_load(ps3->ret_any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                    const DevState s = pstate(ps3, k + pa.swap0);
+                    const int w = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6), W = gridDim.x * (BLOCK / 64);
                     if constexpr (MIXED) ret_walk(s, w, W, [&](int t) { pass_c_ret_mixed_call(s, t); });
                     else ret_walk(s, w, W, [&](int t) { pass_c_ret_call(s, t); });
                 }
