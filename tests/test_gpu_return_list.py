@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 import scenarios as SC
+from dynearthsol_amd import abi
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +55,29 @@ def test_long_return_lists_equal_returns_in_place(nelem, segments):
     assert yields > 64 * 2048        # some wavefront has more than 64
     for k in FIELDS:
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("precision", [abi.DES_FP64, abi.DES_MIXED])
+def test_returns_come_and_go(mode, precision):
+    """Steps in which nothing yields before and after steps in which all does:
+    the return kernel's flag is set and cleared each time.  FP64 against the
+    per-function step, mixed against the other launch mode."""
+    from dynearthsol_amd.lib import DesModel
+    m = SC.build("ep3", nelem=1500)
+    print(m.nelem, "elements, launch mode", mode, "precision", precision, flush=True)
+    high = _yielding(m)
+    low = high.copy()
+    low[:, :2] = high[:, 2:3]          # isotropic but for a little shear: far from the yield surface
+    g, h = DesModel(m), DesModel(m)
+    g.set_launch_mode(mode)
+    h.set_launch_mode(1 - mode)
+    for st, yields in ((low, False), (high, True), (low, False), (high, True)):
+        for a in (g, h):
+            a.upload(stress=st, plstrain=np.zeros(m.nelem), delta_plstrain=np.zeros(m.nelem))
+        g.run(1, precision)
+        h.step(1) if precision == abi.DES_FP64 else h.run(1, precision)
+        a, b = g.download(FIELDS), h.download(FIELDS)
+        assert bool((a["plstrain"] > 0).any()) == yields
+        for k in FIELDS:
+            assert np.array_equal(a[k], b[k]), k
