@@ -1825,37 +1825,42 @@ template <int ND, int DEPTH> __global__ __launch_bounds__(BLOCK) void k_pass_b(D
 // sixth of 200 k elements beyond the yield surface pass C took 48.8 us, and
 // takes 19.3 with the segments.)  The counts are written each step for every wavefront
 // that holds an element, and are zero from the allocation on for the others.
-// A wavefront with an entry also sets ret_any, which pass D clears: where
-// nothing yields the return kernel reads that one number and ends (1.7 us;
-// with every wavefront reading its segments' counts 3.2 us, 1.5 of the 41 us
-// that a step of 12 k tets takes).  Every writer stores the same 1.
 __device__ __forceinline__ bool ret_slot(const DevState &s, int e, bool defer, int &k)
 {
     const unsigned long long mask = __ballot(defer);
     const int lane = __lane_id();
-    if (lane == 0) {                                          // lane 0 holds an element if any lane does
-        s.ret_count[e >> 6] = __popcll(mask);
-        if (mask) *s.ret_any = 1;
-    }
+    if (lane == 0) s.ret_count[e >> 6] = __popcll(mask);      // lane 0 holds an element if any lane does
     k = (e & ~63) + __popcll(mask & ((1ull << lane) - 1));
     return defer;
 }
 
-// Every listed return of s, once: walker w of W wavefronts takes the segments
-// w, w + W, ... (strided, so that a yielding region spreads over all of them)
-// 64 at a time, sums their counts over the lanes and hands out the entries
-// densely, 64 per round.
-template <class F> __device__ __forceinline__ void ret_walk(const DevState &s, int w, int W, F &&item)
+// Every listed return of E elements, once: walker w of W wavefronts takes the
+// segments w, w + W, ... (strided, so that a yielding region spreads over all of
+// them) 64 at a time, sums their counts over the lanes and hands out the entries
+// densely, 64 per round.  Where a walker has at most one segment (up to 131 k
+// elements in 2048 wavefronts) its count is one scalar load and needs no sums:
+// us a step of 12 k and 50 k tets with nothing listed 41.0 -> 39.6 and 42.9 ->
+// 41.0, a sixth listed 47.6 -> 46.7 and 53.5 -> 52.5.  (A flag that says whether
+// anything is listed saves another 1.3 us at 150 k and 300 k tets with nothing
+// listed, and costs 0.5-1 us wherever something is.)
+template <class F> __device__ __forceinline__ void ret_walk(const int *count, int E, int w, int W, F &&item)
 {
     const int lane = __lane_id();
-    const int nseg = (s.E + 63) >> 6;
+    const int nseg = (E + 63) >> 6;
+    w = __builtin_amdgcn_readfirstlane(w);
+    const bool one = W >= nseg;
+    int n = 0;
+    if (one && (w >= nseg || !(n = count[w]))) return;
     for (long c = w; c < nseg; c += 64L * W) {
         const long seg = c + (long)lane * W;
-        int incl = seg < nseg ? s.ret_count[seg] : 0;
+        int incl = n;
+        if (!one) {
+            incl = seg < nseg ? count[seg] : 0;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int v = __shfl_up(incl, d);
-            if (lane >= d) incl += v;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int v = __shfl_up(incl, d);
+                if (lane >= d) incl += v;
+            }
         }
         const int total = __shfl(incl, 63);
         for (int t0 = 0; t0 < total; t0 += 64) {
@@ -2063,7 +2068,7 @@ __device__ __forceinline__ void pass_c_ret_item(const DevState &s, int k)
 
 __global__ __launch_bounds__(64) void k_pass_c_ret(DevState s)
 {
-    if (*s.ret_any) ret_walk(s, blockIdx.x, gridDim.x, [&](int k) { pass_c_ret_item(s, k); });
+    ret_walk(s.ret_count, s.E, blockIdx.x, gridDim.x, [&](int k) { pass_c_ret_item(s, k); });
 }
 
 // pass D: node sum of dp * volume (NMD_stress, geometry.cxx:203-216)
@@ -2094,7 +2099,6 @@ template <int ND, int NB, int DEPTH> __device__ __forceinline__ void pass_d_body
 
 template <int ND, int NB, int DEPTH = 4> __global__ __launch_bounds__(NB) void k_pass_d(DevState s, FusedFlags fl)
 {
-    if (ND == 3 && blockIdx.x == 0 && threadIdx.x == 0) *s.ret_any = 0;      // for the next step's pass C
     pass_d_body<ND, NB, DEPTH>(s, fl, xcd_block(s.rev));
 }
 
@@ -2493,7 +2497,7 @@ __device__ __forceinline__ void pass_c_ret_mixed_item(const DevState &s, int k)
 
 __global__ __launch_bounds__(64) void k_pass_c_ret_mixed(DevState s)
 {
-    if (*s.ret_any) ret_walk(s, blockIdx.x, gridDim.x, [&](int k) { pass_c_ret_mixed_item(s, k); });
+    ret_walk(s.ret_count, s.E, blockIdx.x, gridDim.x, [&](int k) { pass_c_ret_mixed_item(s, k); });
 }
 
 template <int ND> __device__ __forceinline__ void pass_e_mixed_body(DevState s, const FusedFlags &fl, int blk,
@@ -2703,17 +2707,15 @@ __global__ __launch_bounds__(BLOCK, 2) void k_persistent(const DevState *__restr
             if (g3.plastic) {       // the deferred Mohr-Coulomb returns (3D only)
                 // the calls take the state in scratch: copied there only where
                 // there is a call (3D, 12 k tets: 4.0 -> 3.6 ms for 50 steps)
-                if (__hip_atomic_load(ps3->ret_any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                const int w = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6), W = gridDim.x * (BLOCK / 64);
+                ret_walk(ps3->ret_count, ps3->E, w, W, [&](int t) {
                     const DevState s = pstate(ps3, k + pa.swap0);
-                    const int w = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6), W = gridDim.x * (BLOCK / 64);
-                    if constexpr (MIXED) ret_walk(s, w, W, [&](int t) { pass_c_ret_mixed_call(s, t); });
-                    else ret_walk(s, w, W, [&](int t) { pass_c_ret_call(s, t); });
-                }
+                    if constexpr (MIXED) pass_c_ret_mixed_call(s, t);
+                    else pass_c_ret_call(s, t);
+                });
                 grid.sync();
             }
         }
-        if constexpr (HAS3)
-            if (blockIdx.x == 0 && threadIdx.x == 0) *ps3->ret_any = 0;      // for the next step's pass C
         PWALK(nn3, nn2, pa.rev, (pass_d_body<3, BLOCK, 8>(s, fl, b)), (pass_d_body<2, BLOCK, 8>(s, fl, b)));
         grid.sync();
         if constexpr (MIXED)
@@ -4394,7 +4396,6 @@ int ensure_retlist(des_ctx *ctx)
     const size_t nseg = ((size_t)ctx->E + 63) / 64;      // one list segment per wavefront of elements
     if ((rc = dalloc_n(ctx, &s.ret_elem, nseg * 64))) return rc;
     if ((rc = dalloc_n(ctx, &s.ret_val, nseg * 64 * 8))) return rc;
-    if ((rc = dalloc_n(ctx, &s.ret_any, 1))) return rc;
     if ((rc = dalloc_n(ctx, &s.ret_count, nseg))) return rc;
     return DES_OK;
 }

@@ -115,8 +115,8 @@ struct DevState {
     // elements whose Mohr-Coulomb return is left to the return kernel of the
     // fused schedule, in segments of 64 (element e's is e / 64): each
     // segment's count, element ids, and per entry the trial stress and the
-    // stress trace before the update (8 doubles); ret_any: some count is not 0
-    int *ret_any, *ret_count, *ret_elem;
+    // stress trace before the update (8 doubles)
+    int *ret_count, *ret_elem;
     double *ret_val;
     MixedRet *ret_mix;                            // the mixed-precision schedule's records
     // node records of the fused schedule (NREC doubles per node): x[ND],

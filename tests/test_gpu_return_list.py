@@ -61,8 +61,8 @@ def test_long_return_lists_equal_returns_in_place(nelem, segments):
 @pytest.mark.parametrize("precision", [abi.DES_FP64, abi.DES_MIXED])
 def test_returns_come_and_go(mode, precision):
     """Steps in which nothing yields before and after steps in which all does:
-    the return kernel's flag is set and cleared each time.  FP64 against the
-    per-function step, mixed against the other launch mode."""
+    the lists fill and empty each time.  FP64 against the per-function step,
+    mixed against the other launch mode."""
     from dynearthsol_amd.lib import DesModel
     m = SC.build("ep3", nelem=1500)
     print(m.nelem, "elements, launch mode", mode, "precision", precision, flush=True)
